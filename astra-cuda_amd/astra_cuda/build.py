@@ -9,10 +9,12 @@ torch, it binds to the runtime torch already loaded, so both share streams.
 """
 from __future__ import annotations
 
+import concurrent.futures
 import os
 import shutil
 import subprocess
 import sys
+import tempfile
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(os.path.dirname(PKG_DIR))
@@ -24,12 +26,17 @@ SOURCES = [os.path.join(CSRC, "market.hip"), os.path.join(CSRC, "high_low.hip")]
 
 ARCH = os.environ.get("ASTRA_OFFLOAD_ARCH", "gfx950")
 
+# market.hip's kernels are templates of the number of 64-level mask words: one unit
+# for each, and one for the entry points, compiled side by side.
+UNITS = [("market", SOURCES[0], ["-DASTRA_W_UNITS"])] + \
+        [(f"market_w{w}", SOURCES[0], [f"-DASTRA_W={w}"]) for w in (16, 8, 4, 2, 1)] + \
+        [("high_low", SOURCES[1], [])]
+
 HIPCC_FLAGS = [
     f"--offload-arch={ARCH}",
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     "-mcode-object-version=5",
     # keep the compiler from emitting packed FP32 ops (unused here anyway)
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -85,14 +92,23 @@ def build_binding(verbose: bool = False) -> str:
 def build(verbose: bool = False) -> str:
     """Compile the sources into the package directory. Always recompiles."""
     tmp = LIB_PATH + ".tmp"
-    cmd = [hipcc(), *HIPCC_FLAGS, f"-I{INCLUDE}", *SOURCES, "-o", tmp]
+    with tempfile.TemporaryDirectory() as d:
+        objs = [os.path.join(d, name + ".o") for name, _, _ in UNITS]
+        cmds = [[hipcc(), *HIPCC_FLAGS, *flags, f"-I{INCLUDE}", "-c", src, "-o", obj]
+                for (_, src, flags), obj in zip(UNITS, objs)]
+        with concurrent.futures.ThreadPoolExecutor(min(len(cmds), os.cpu_count() or 1)) as pool:
+            list(pool.map(lambda c: _run(c, verbose), cmds))
+        _run([hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp], verbose)
+    os.replace(tmp, LIB_PATH)
+    return LIB_PATH
+
+
+def _run(cmd: list, verbose: bool) -> None:
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed ({res.returncode}):\n{res.stdout}\n{res.stderr}")
-    os.replace(tmp, LIB_PATH)
-    return LIB_PATH
 
 
 if __name__ == "__main__":

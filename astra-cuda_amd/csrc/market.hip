@@ -2428,19 +2428,6 @@ int launch_quote_match(const astra_market *h, const QuoteIn &in, const FillOut &
   return ASTRA_OK;
 }
 
-int launch_bbo(const astra_market *h, int32_t *bp, int32_t *bs, int32_t *ap, int32_t *as,
-               hipStream_t s) {
-  const Book b = book_of(h);
-#ifdef ASTRA_HOST_EMULATION
-  (void)s;
-  for (int64_t m = 0; m < b.M; ++m) bbo_copy_market(b, bp, bs, ap, as, m);
-#else
-  hipLaunchKernelGGL(bbo_kernel, dim3(grid_for(b.M, 256)), dim3(256), 0, s, b, bp, bs, ap, as);
-#endif
-  ASTRA_HIP_CHECK(rt_last_error(), "GetBBOs");
-  return ASTRA_OK;
-}
-
 template <int W>
 int launch_clear_quotes(const astra_market *h, const uint8_t *reset, hipStream_t s) {
   const Book b = book_of(h);
@@ -2456,32 +2443,80 @@ int launch_clear_quotes(const astra_market *h, const uint8_t *reset, hipStream_t
   return ASTRA_OK;
 }
 
-template <int W>
-int launch_quote_match_plain(const astra_market *h, const QuoteIn &in, const FillOut &fo,
-                             hipStream_t s) {
-  return launch_quote_match<W, false, false>(h, in, fo, StepOut{}, 1, s);
-}
+// One launch that depends on the number of mask words W, as the entry points ask for it.
+enum class CallKind { kQuotes, kGameMove, kSteps, kClear };
+struct Call {
+  CallKind kind;
+  const astra_market *h;
+  const QuoteIn *in;
+  const FillOut *out;
+  const StepOut *steps_out;
+  int32_t steps;
+  const uint8_t *reset;
+  hipStream_t stream;
+};
 
 template <int W>
-int launch_quote_match_game(const astra_market *h, const QuoteIn &in, const FillOut &fo,
-                            hipStream_t s) {
-  return launch_quote_match<W, true, false>(h, in, fo, StepOut{}, 1, s);
-}
-
-template <int W>
-int launch_quote_match_steps(const astra_market *h, const QuoteIn &in, const FillOut &fo,
-                             const StepOut &so, int32_t steps, hipStream_t s) {
-  return launch_quote_match<W, false, true>(h, in, fo, so, steps, s);
-}
-
-#define ASTRA_DISPATCH_W(W_, FN, ...)  \
-  switch (W_) {                        \
-    case 1: return FN<1>(__VA_ARGS__); \
-    case 2: return FN<2>(__VA_ARGS__); \
-    case 4: return FN<4>(__VA_ARGS__); \
-    case 8: return FN<8>(__VA_ARGS__); \
-    default: return FN<16>(__VA_ARGS__); \
+int launch_call(const Call &c) {
+  switch (c.kind) {
+    case CallKind::kQuotes:
+      return launch_quote_match<W, false, false>(c.h, *c.in, *c.out, StepOut{}, 1, c.stream);
+    case CallKind::kGameMove:
+      return launch_quote_match<W, true, false>(c.h, *c.in, *c.out, StepOut{}, 1, c.stream);
+    case CallKind::kSteps:
+      return launch_quote_match<W, false, true>(c.h, *c.in, *c.out, *c.steps_out, c.steps, c.stream);
+    default:
+      return launch_clear_quotes<W>(c.h, c.reset, c.stream);
   }
+}
+
+#if defined(ASTRA_W)
+}  // namespace
+
+// This unit holds the kernels of ASTRA_W mask words only: the build compiles one
+// such unit per W beside the unit of the entry points, all at once.
+#define ASTRA_CAT2(a, b) a##b
+#define ASTRA_CAT(a, b) ASTRA_CAT2(a, b)
+__attribute__((visibility("hidden"))) int ASTRA_CAT(astra_launch_call_w, ASTRA_W)(const void *call) {
+  return launch_call<ASTRA_W>(*static_cast<const Call *>(call));
+}
+#else
+
+#if defined(ASTRA_W_UNITS)
+}  // namespace
+int astra_launch_call_w1(const void *call);
+int astra_launch_call_w2(const void *call);
+int astra_launch_call_w4(const void *call);
+int astra_launch_call_w8(const void *call);
+int astra_launch_call_w16(const void *call);
+namespace {
+#define ASTRA_CALL_W(W_) astra_launch_call_w##W_(&c)
+#else
+#define ASTRA_CALL_W(W_) launch_call<W_>(c)
+#endif
+
+int launch_for_levels(const Call &c) {
+  switch (c.h->lay.W) {
+    case 1: return ASTRA_CALL_W(1);
+    case 2: return ASTRA_CALL_W(2);
+    case 4: return ASTRA_CALL_W(4);
+    case 8: return ASTRA_CALL_W(8);
+    default: return ASTRA_CALL_W(16);
+  }
+}
+
+int launch_bbo(const astra_market *h, int32_t *bp, int32_t *bs, int32_t *ap, int32_t *as,
+               hipStream_t s) {
+  const Book b = book_of(h);
+#ifdef ASTRA_HOST_EMULATION
+  (void)s;
+  for (int64_t m = 0; m < b.M; ++m) bbo_copy_market(b, bp, bs, ap, as, m);
+#else
+  hipLaunchKernelGGL(bbo_kernel, dim3(grid_for(b.M, 256)), dim3(256), 0, s, b, bp, bs, ap, as);
+#endif
+  ASTRA_HIP_CHECK(rt_last_error(), "GetBBOs");
+  return ASTRA_OK;
+}
 
 int launch_fill(void *dst, int64_t n_words, uint32_t v, hipStream_t s, const char *what) {
   if (n_words <= 0) return ASTRA_OK;
@@ -2772,8 +2807,8 @@ int astra_market_add_two_sided_quotes(astra_market *h, const int32_t *bid_px,
     const FillOut fo{fill_prices,        fill_sizes,       fill_customer_ids, fill_quoter_ids,
                      fill_is_sell_quote, fill_quote_sizes, fill_tid,          fill_quote_tid,
                      fill_counts,        nullptr};
-    // (returns; the kernel moves the TID counter on by 2, market.cu:531)
-    ASTRA_DISPATCH_W(h->lay.W, launch_quote_match_plain, h, in, fo, as_stream(stream));
+    // (the kernel moves the TID counter on by 2, market.cu:531)
+    return launch_for_levels({CallKind::kQuotes, h, &in, &fo, nullptr, 1, nullptr, as_stream(stream)});
   }
   DeviceGuard g(h->device);
   return advance_tid_empty(h, 2, as_stream(stream));
@@ -2796,8 +2831,8 @@ int astra_market_add_two_sided_quotes_rows(astra_market *h, const int32_t *bid_p
     FillOut fo{};
     fo.counts = fill_counts;
     fo.rows = fill_rows;
-    // (returns; the kernel moves the TID counter on by 2, market.cu:531)
-    ASTRA_DISPATCH_W(h->lay.W, launch_quote_match_plain, h, in, fo, as_stream(stream));
+    // (the kernel moves the TID counter on by 2, market.cu:531)
+    return launch_for_levels({CallKind::kQuotes, h, &in, &fo, nullptr, 1, nullptr, as_stream(stream)});
   }
   DeviceGuard g(h->device);
   return advance_tid_empty(h, 2, as_stream(stream));
@@ -2838,8 +2873,8 @@ int astra_market_add_two_sided_quotes_steps(
     StepOut so{};
     so.counts = step_fill_counts;
     so.bbo[0] = step_bbos;  // step_views derives the other three fields' rows
-    // (returns; the kernel moves the TID counter on by 2 per step, market.cu:531)
-    ASTRA_DISPATCH_W(h->lay.W, launch_quote_match_steps, h, in, fo, so, steps, as_stream(stream));
+    // (the kernel moves the TID counter on by 2 per step, market.cu:531)
+    return launch_for_levels({CallKind::kSteps, h, &in, &fo, &so, steps, nullptr, as_stream(stream)});
   }
   DeviceGuard g(h->device);
   return advance_tid_empty(h, (int32_t)(2u * (uint32_t)steps), as_stream(stream));
@@ -2873,9 +2908,9 @@ int astra_game_move(astra_market *h, const GameMove &g, int32_t *const fill_fiel
       fo.tid = fill_fields[6];
       fo.quote_tid = fill_fields[7];
     }
-    // (returns; the kernel moves the TID counter on by 2, market.cu:531,
+    // (the kernel moves the TID counter on by 2, market.cu:531,
     // unless the move's checks failed)
-    ASTRA_DISPATCH_W(h->lay.W, launch_quote_match_game, h, in, fo, stream);
+    return launch_for_levels({CallKind::kGameMove, h, &in, &fo, nullptr, 1, nullptr, stream});
   }
   DeviceGuard dg(h->device);
   return advance_tid_empty(h, 2, stream);
@@ -2931,7 +2966,7 @@ int astra_market_clear_quotes(astra_market *h, const uint8_t *reset, void *strea
   if (h->M == 0) return ASTRA_OK;
   if (!reset) return fail(ASTRA_ERR_INVALID_ARGUMENT, "NULL reset mask");
   DeviceGuard g(h->device);
-  ASTRA_DISPATCH_W(h->lay.W, launch_clear_quotes, h, reset, as_stream(stream));
+  return launch_for_levels({CallKind::kClear, h, nullptr, nullptr, nullptr, 1, reset, as_stream(stream)});
 }
 
 int astra_market_portfolios(const astra_market *h, int32_t **p) {
@@ -3035,3 +3070,4 @@ int astra_market_set_tid(astra_market *h, int32_t tid, void *stream) {
 }
 
 }  // extern "C"
+#endif  // ASTRA_W

@@ -15,7 +15,9 @@
 //    chains at once.
 //  * Per market and side, the occupancy of the L price levels is a bitmask of
 //    W = ceil(L/64) 64-bit words kept in registers during a call; bit p is set
-//    exactly when the level's head is not NULL. Best bid / best ask are
+//    exactly when the level has a list. A level's word is read only where its bit
+//    is set, so an emptied level (and a cleared book) writes no NULL: one scattered
+//    write less per emptied level. Best bid / best ask are
 //    count-leading/trailing-zeros over the mask, replacing the reference's
 //    O(L) rescans. The masks live in HBM as structure-of-arrays
 //    mask[side][word][market], so their loads and stores are fully coalesced.
@@ -305,6 +307,23 @@ template <int W>
 ASTRA_HD void mask_clear(uint64_t (&m)[W], int p) {
 #pragma unroll
   for (int i = 0; i < W; ++i) m[i] &= ~((uint64_t)((p >> 6) == i) << (p & 63));
+}
+
+// 0 if bit p is set, else all ones (also for a p outside the mask).
+template <int W>
+ASTRA_HD uint32_t mask_absent(const uint64_t (&m)[W], int p) {
+  uint64_t r = 0;
+#pragma unroll
+  for (int i = 0; i < W; ++i) r |= (p >> 6) == i ? m[i] : 0ull;
+  return (uint32_t)((r >> (p & 63)) & 1ull) - 1u;
+}
+
+// The value, computed at this point of the program and not later.
+ASTRA_HD uint32_t pinned(uint32_t v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(v));
+#endif
+  return v;
 }
 
 // Byte offsets of one side's {head, tail} pair within a level: side 0 = bid, 1 = ask.
@@ -646,12 +665,10 @@ struct GlobalBook {
   uint4 *rec;
   ASTRA_HD uint4 record(uint32_t s) const { return rec[s]; }
   ASTRA_HD int32_t size(uint32_t s) const { return reinterpret_cast<const int32_t *>(rec + s)[0]; }
-  ASTRA_HD uint32_t word(int32_t p, int side) const { return level_word(lv, p, side); }
   ASTRA_HD uint32_t head(int32_t p, int side) const { return level_head(lv, p, side); }
   ASTRA_HD void set_size(uint32_t s, int32_t v) const {
     reinterpret_cast<int32_t *>(rec + s)[0] = v;
   }
-  ASTRA_HD void set_word(int32_t p, int side, uint32_t w) const { store_level_word(lv, p, side, w); }
   ASTRA_HD void set_head(int32_t p, int side, uint32_t h) const { store_head(lv, p, side, h); }
 };
 
@@ -664,15 +681,10 @@ struct StagedBook {
   uint4 *grec;
   ASTRA_HD uint4 record(uint32_t s) const { return srec[s]; }
   ASTRA_HD int32_t size(uint32_t s) const { return reinterpret_cast<const int32_t *>(srec + s)[0]; }
-  ASTRA_HD uint32_t word(int32_t p, int side) const { return level_word(slv, p, side); }
   ASTRA_HD uint32_t head(int32_t p, int side) const { return level_head(slv, p, side); }
   ASTRA_HD void set_size(uint32_t s, int32_t v) const {
     reinterpret_cast<int32_t *>(srec + s)[0] = v;
     gst(reinterpret_cast<int32_t *>(grec + s), v);
-  }
-  ASTRA_HD void set_word(int32_t p, int side, uint32_t w) const {
-    store_level_word(slv, p, side, w);
-    gst(reinterpret_cast<uint32_t *>(glv + (size_t)p * 4 + 2 * side), w);
   }
   ASTRA_HD void set_head(int32_t p, int side, uint32_t h) const {
     store_head(slv, p, side, h);
@@ -706,7 +718,6 @@ struct UniformStagedBook : StagedBook {
   ASTRA_HD int32_t size(uint32_t s) const {
     return uni(reinterpret_cast<const int32_t *>(srec + s)[0]);
   }
-  ASTRA_HD uint32_t word(int32_t p, int side) const { return uni(level_word(slv, p, side)); }
   ASTRA_HD uint32_t head(int32_t p, int side) const { return uni(level_head(slv, p, side)); }
 };
 
@@ -1050,14 +1061,26 @@ ASTRA_HD void quote_prologue(const Book &b, const QuoteIn &in, int64_t m, Market
   const uint32_t hb0 = hb0f == kNull16 ? kNull16 : (hb0f & ~kSizeKnown);
   const uint32_t ha0 = ha0f == kNull16 ? kNull16 : (ha0f & ~kSizeKnown);
 
+  // An empty level's word is stale: its mask bit makes it NULL. OR-ed in, not
+  // selected: the compiler turns a select into a branch around the load; and made
+  // here, while the masks are at hand, not behind the second round trip. A pop that
+  // empties a level and ClearQuotes then store no NULL word (one scattered write of
+  // about 17 per market and step less; large launches are bound by such requests).
+  // Steps of one state after another, past the ring's wrap: 524,288 markets 371 ->
+  // 360 us, 16 steps of 100,000 in one launch (row layout) 626 -> 611, 32 of 10,000
+  // 357 -> 350, 100,000 markets 65.8 -> 63.5 (with the select 68.7, with the OR behind
+  // the second round trip 66.7) and unchanged where states alternate.
+  const uint32_t bnone = pinned(mask_absent<W>(s.bm, bid_px));
+  const uint32_t anone = pinned(mask_absent<W>(s.am, ask_px));
+
   // ---- round trip 2 ----
   // The insert levels' words: unconditional loads (level 0 stands in for a
   // rejected quote) so that nothing waits on them before the loads below are
   // issued; conditional ones each cost a round trip of their own.
   const uint32_t bword_ld = level_word(lv, bid_ok ? bid_px : 0, 0);
   const uint32_t aword_ld = level_word(lv, ask_ok ? ask_px : 0, 1);
-  const uint32_t bword = bid_ok ? bword_ld : 0u;
-  const uint32_t aword = ask_ok ? aword_ld : 0u;
+  const uint32_t bword = bid_ok ? (bword_ld | bnone) : 0u;
+  const uint32_t aword = ask_ok ? (aword_ld | anone) : 0u;
   uint4 hrb = make_uint4((uint32_t)bsz0, 0, 0, 0), hra = make_uint4((uint32_t)asz0, 0, 0, 0);
   // Head records read here: a crossing book's, all where the call hands out the
   // BBO, and a head whose size the cache does not hold (so that this call's
@@ -1242,7 +1265,6 @@ ASTRA_HD bool zero_levels(LoopState<W> &s, const MarketCtx &c, const BookMem &bk
       ++s.npass;
       ++s.emptied;
     }
-    bk.set_word(p, SIDE, 0xFFFFFFFFu);
     mask_clear<W>(m, p);
     p = SIDE == 0 ? mask_highest<W>(m) : mask_lowest<W>(m, L);
     const bool live = SIDE == 0 ? p >= 0 : p < L;
@@ -1303,7 +1325,7 @@ ASTRA_HD bool cross_run(LoopState<W> &s, const MarketCtx &c, const BookMem &bk, 
     if (pop_b) {
       bk.set_size(s.bh, 0);
       if (nb == kNull16) {
-        bk.set_word(s.bb, 0, 0xFFFFFFFFu);
+        if (head_b) bk.set_head(s.bb, 0, s.bh);  // what the passes one by one leave
         head_b = false;
         mask_clear<W>(s.bm, s.bb);
         if (STATS) ++s.emptied;
@@ -1319,7 +1341,7 @@ ASTRA_HD bool cross_run(LoopState<W> &s, const MarketCtx &c, const BookMem &bk, 
     if (pop_a) {
       bk.set_size(s.ah, 0);
       if (na == kNull16) {
-        bk.set_word(s.ba, 1, 0xFFFFFFFFu);
+        if (head_a) bk.set_head(s.ba, 1, s.ah);  // what the passes one by one leave
         head_a = false;
         mask_clear<W>(s.am, s.ba);
         if (STATS) ++s.emptied;
@@ -1518,7 +1540,6 @@ ASTRA_HD bool match_loop(LoopState<W> &s, const MarketCtx &c, const BookMem &bk,
     if (s.brec.x == 0u) {  // pop the bid head (:241-256)
       const uint32_t nh = rec_next(s.brec);
       if (nh == kNull16) {
-        bk.set_word(s.bb, 0, 0xFFFFFFFFu);
         mask_clear<W>(s.bm, s.bb);
         if (STATS) ++s.emptied;
         if constexpr (BookMem::kStaged) {  // the highest remaining level and its head
@@ -1542,7 +1563,6 @@ ASTRA_HD bool match_loop(LoopState<W> &s, const MarketCtx &c, const BookMem &bk,
     if (s.arec.x == 0u) {  // pop the ask head (:258-273)
       const uint32_t nh = rec_next(s.arec);
       if (nh == kNull16) {
-        bk.set_word(s.ba, 1, 0xFFFFFFFFu);
         mask_clear<W>(s.am, s.ba);
         if (STATS) ++s.emptied;
         if constexpr (BookMem::kStaged) {  // the lowest remaining level and its head
@@ -1722,29 +1742,22 @@ ASTRA_HD void last_price_market(int32_t *last, const int32_t *counts, const int3
   if (c > 0 && c <= F) last[m] = prices[(m * (int64_t)F + (c - 1)) * stride];
 }
 
-// ClearQuotes (market.cu:735-749) for thread t = (market, level): the level's
-// 8-byte word to all-NULL; the level-0 thread also zeroes the masks and the slot
-// counter and empties the market's BBO cache. The reference also writes NULL
-// into order_next; here a slot's next is
+// ClearQuotes (market.cu:735-749) for a selected market: masks and slot counter 0,
+// BBO cache empty. The level words stay as they are: an empty level's word is not
+// read. The reference also writes NULL into order_next; here a slot's next is
 // overwritten whenever the slot is reused, and after the clear no list can
 // reach a slot that was not reused, so it is left alone (no observable
 // difference).
 template <int W>
-ASTRA_HD void clear_quotes_thread(const Book &b, const uint8_t *reset, int64_t t) {
-  const int64_t per = b.L > 0 ? b.L : 1;
-  const int64_t m = t / per;
-  const int64_t p = t - m * per;
-  if (m >= b.M || !reset[m]) return;
+ASTRA_HD void clear_quotes_market(const Book &b, const uint8_t *reset, int64_t m) {
+  if (!reset[m]) return;
   const int64_t M = b.M;
-  if (p < b.L) reinterpret_cast<uint64_t *>(b.levels)[m * (int64_t)b.L + p] = ~0ull;
-  if (p == 0) {
 #pragma unroll
-    for (int i = 0; i < 2 * W; ++i) b.masks[(int64_t)i * M + m] = 0ull;
-    b.next_slot[m] = 0;
-    b.bbo[m] = ASTRA_NULL_INDEX;
-    b.bbo[M + m] = ASTRA_NULL_INDEX;
-    b.tob[m] = 0xFFFFFFFFu;
-  }
+  for (int i = 0; i < 2 * W; ++i) b.masks[(int64_t)i * M + m] = 0ull;
+  b.next_slot[m] = 0;
+  b.bbo[m] = ASTRA_NULL_INDEX;
+  b.bbo[M + m] = ASTRA_NULL_INDEX;
+  b.tob[m] = 0xFFFFFFFFu;
 }
 
 // ---- __global__ wrappers ----
@@ -2200,11 +2213,13 @@ __global__ __launch_bounds__(256) void last_price_kernel(int32_t *last, const in
   if (m < M) last_price_market(last, counts, prices, F, stride, m);
 }
 
+// One lane per market, coalesced words only (a lane per level, with a 64-bit division
+// to find its market, made a step of 30,000 markets with 1/64 of them cleared 39.7 us;
+// 33.4 us now).
 template <int W>
-__global__ __launch_bounds__(256) void clear_quotes_kernel(Book b, const uint8_t *reset,
-                                                           int64_t n) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) clear_quotes_thread<W>(b, reset, t);
+__global__ __launch_bounds__(256) void clear_quotes_kernel(Book b, const uint8_t *reset) {
+  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (m < b.M) clear_quotes_market<W>(b, reset, m);
 }
 
 // Grid-stride fill of n 32-bit words; 16-byte stores when dst is 16-byte aligned.
@@ -2431,13 +2446,11 @@ int launch_quote_match(const astra_market *h, const QuoteIn &in, const FillOut &
 template <int W>
 int launch_clear_quotes(const astra_market *h, const uint8_t *reset, hipStream_t s) {
   const Book b = book_of(h);
-  const int64_t n = (int64_t)std::max<int32_t>(h->L, 1) * h->M;
 #ifdef ASTRA_HOST_EMULATION
   (void)s;
-  for (int64_t t = 0; t < n; ++t) clear_quotes_thread<W>(b, reset, t);
+  for (int64_t m = 0; m < b.M; ++m) clear_quotes_market<W>(b, reset, m);
 #else
-  hipLaunchKernelGGL((clear_quotes_kernel<W>), dim3(grid_for(n, 256)), dim3(256), 0, s, b, reset,
-                     n);
+  hipLaunchKernelGGL((clear_quotes_kernel<W>), dim3(grid_for(b.M, 256)), dim3(256), 0, s, b, reset);
 #endif
   ASTRA_HIP_CHECK(rt_last_error(), "ClearQuotes");
   return ASTRA_OK;
@@ -2999,6 +3012,7 @@ int astra_market_to_string(const astra_market *h, int32_t market_id, char *buf, 
     DeviceGuard g(h->device);
     std::vector<uint16_t> lv((size_t)h->L * 4);
     std::vector<uint4> rec((size_t)h->O);
+    std::vector<uint64_t> masks((size_t)2 * h->lay.W);
     hipStream_t st = as_stream(stream);
     if (h->L > 0)
       ASTRA_HIP_CHECK(rt_memcpy(lv.data(), h->ws + h->lay.levels + (size_t)market_id * h->L * 8,
@@ -3007,14 +3021,21 @@ int astra_market_to_string(const astra_market *h, int32_t market_id, char *buf, 
     ASTRA_HIP_CHECK(rt_memcpy(rec.data(), h->ws + h->lay.records + (size_t)market_id * h->O * 16,
                               (size_t)h->O * 16, st),
                     "ToString");
+    for (size_t i = 0; i < masks.size(); ++i)
+      ASTRA_HIP_CHECK(rt_memcpy(&masks[i], h->ws + h->lay.masks + (i * h->M + market_id) * 8, 8, st),
+                      "ToString");
     ASTRA_HIP_CHECK(rt_sync(st), "ToString");
     std::vector<Row> sells, buys;
-    for (int32_t p = 0; p < h->L; ++p) walk_level(rec, lv[(size_t)p * 4 + 2], p, h->O, sells);
+    // the head of level p's list on `side`: its word counts where the mask bit is set
+    auto head = [&](int32_t p, int side) -> uint32_t {
+      return (masks[(size_t)(side * h->lay.W + p / 64)] >> (p % 64)) & 1 ? lv[(size_t)p * 4 + 2 * side] : kNull16;
+    };
+    for (int32_t p = 0; p < h->L; ++p) walk_level(rec, head(p, 1), p, h->O, sells);
     std::sort(sells.begin(), sells.end(), [](const Row &a, const Row &b) {  // :645-651
       if (a.price != b.price) return a.price > b.price;
       return a.tid < b.tid;
     });
-    for (int32_t p = h->L - 1; p >= 0; --p) walk_level(rec, lv[(size_t)p * 4], p, h->O, buys);
+    for (int32_t p = h->L - 1; p >= 0; --p) walk_level(rec, head(p, 0), p, h->O, buys);
     std::snprintf(line, sizeof line, "####### %zu sell orders #######\n", sells.size());  // :677
     s += line;
     for (const Row &r : sells) {

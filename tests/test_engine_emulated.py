@@ -210,6 +210,37 @@ def test_emulated_reset_clear_clone_to_string():
     assert np.array_equal(em.portfolios, om.customer_portfolios)
 
 
+@pytest.mark.parametrize("L", [1, 64, 65, 129, 513])
+def test_emulated_emptied_and_cleared_levels_start_anew(L):
+    """Levels that empty, are cleared and fill again, at the mask words' edges: an empty
+    level's word is never NULLed, so only its mask bit may decide (whole numbers: exact)."""
+    M, O, F, C = 33, 24, 30, 3
+    rng = np.random.default_rng(L)
+    e, o = EmuMarket(M, L, O, F, C, extended=True), OracleMarket(M, L, O, F, C)
+    ef, of = e.new_fill_batch(), o.new_fill_batch()
+    eb, ob = e.new_bbo_batch(), o.new_bbo_batch()
+    edges = np.unique(np.clip([0, 1, 62, 63, 64, 65, 127, 128, 511, 512, L - 2, L - 1], 0, L - 1))
+    for t in range(200):
+        px = [rng.choice(edges, M).astype(np.int32) for _ in range(2)]
+        sz = [rng.integers(0, 4, M).astype(np.int32) for _ in range(2)]
+        args = (px[0], sz[0], px[1], sz[1], rng.integers(0, C, M).astype(np.int32))
+        e.add_two_sided_quotes(*args, ef)
+        o.add_two_sided_quotes(*args, of)
+        if t % 5 == 3:
+            mask = rng.random(M) < 0.4
+            e.clear_quotes(mask)
+            o.clear_quotes(mask)
+        if t == 120:
+            e.reset()
+            o.reset()
+        e.get_bbos(eb)
+        o.get_bbos(ob)
+        _compare(e, ef, eb, o, of, ob, F, f"L={L} step {t}")
+        if t % 9 == 0:
+            for m in range(0, M, 4):
+                assert e.to_string(m) == o.to_string(m), (L, t, m)
+
+
 def test_emulated_zero_sized_shapes():
     # M = 0 and F = 0 and L = 0 are accepted by the reference constructor
     em = EmuMarket(0, 128, 16, 16, 4)

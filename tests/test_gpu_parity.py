@@ -309,6 +309,43 @@ def test_gpu_reset_clear_clone_and_to_string():
     compare_portfolios(g, o, "original after clone")
 
 
+@pytest.mark.parametrize("M", [1, 64, 257, 4000])
+@pytest.mark.parametrize("L", [1, 64, 65, 129, 513])
+def test_gpu_emptied_and_cleared_levels_start_anew(L, M):
+    """Levels that empty, are cleared and fill again, at the mask words' and the clearing
+    workgroups' edges: an empty level's word is never NULLed, so only its mask bit may
+    decide (whole numbers: exact)."""
+    from oracle.oracle import OracleMarket
+    from astra_cuda import order_matching as aom
+    O, F, C = 24, 30, 3
+    rng = np.random.default_rng(L * 7 + M)
+    g = aom.VecMarket(M, L, O, F, C, allow_extended_shapes=True)
+    o = OracleMarket(M, L, O, F, C)
+    gf, of = g.new_fill_batch(), o.new_fill_batch()
+    gb, ob = g.new_bbo_batch(), o.new_bbo_batch()
+    edges = np.unique(np.clip([0, 1, 62, 63, 64, 65, 127, 128, 511, 512, L - 2, L - 1], 0, L - 1))
+    for t in range(60):
+        px = [rng.choice(edges, M).astype(np.int32) for _ in range(2)]
+        sz = [rng.integers(0, 4, M).astype(np.int32) for _ in range(2)]
+        args = (px[0], sz[0], px[1], sz[1], rng.integers(0, C, M).astype(np.int32))
+        g.add_two_sided_quotes(*(t32(a) for a in args), gf)
+        o.add_two_sided_quotes(*args, of)
+        compare_fills(gf, of, F, f"L={L} M={M} step {t}")
+        if t % 5 == 3:
+            mask = rng.random(M) < 0.4
+            g.clear_quotes(torch.as_tensor(mask).to(DEV))
+            o.clear_quotes(mask)
+        if t == 40:
+            g.reset()
+            o.reset()
+        if t % 5 == 4:
+            g.get_bbos(gb)
+            o.get_bbos(ob)
+            compare_bbo(gb, ob, f"L={L} M={M} step {t}")
+            compare_portfolios(g, o, f"L={L} M={M} step {t}")
+            assert g.to_string(M - 1) == o.to_string(M - 1), (L, M, t)
+
+
 def test_gpu_portfolio_view_is_live_and_copy_to():
     from astra_cuda import order_matching as aom
     g = aom.VecMarket(3, 128, 64, 16)

@@ -129,6 +129,14 @@ def test_gpu_game_vs_oracle(N, P, T, S, cM, V, shape, seed, budget, knobs):
     assert not s.market.get_customer_portfolios().any()
 
 
+@pytest.mark.parametrize("per_wave", [16, 64])
+@pytest.mark.parametrize("N,P", [(65, 4), (131, 5), (257, 6), (63, 7), (1, 8), (70, 9)])
+def test_gpu_game_player_counts_ragged(N, P, per_wave):
+    """Each player count the move's rewards are written out for, and the first beyond
+    them, over ragged env counts (whole numbers: exact)."""
+    test_gpu_game_vs_oracle(N, P, 3, 5, 5, 30, None, 20 + P, None, {"per_wave": per_wave})
+
+
 def test_gpu_hand_game():
     g = _game(HAND_GAME["params"])
     s = g.new_initial_state()

@@ -2561,6 +2561,56 @@ int launch_last_price(int32_t *last, const int32_t *counts, const int32_t *price
   return ASTRA_OK;
 }
 
+// Level p of market m as the host reads it: a side whose mask bit is not set is NULL.
+ASTRA_HD uint64_t live_level(const Book &b, int32_t W, int64_t m, int32_t p) {
+  const uint64_t word = reinterpret_cast<const uint64_t *>(b.levels)[m * b.L + p];
+  const uint64_t bid = b.masks[(int64_t)(p >> 6) * b.M + m];
+  const uint64_t ask = b.masks[(int64_t)(W + (p >> 6)) * b.M + m];
+  return word | ((bid >> (p & 63)) & 1 ? 0ull : 0xFFFFFFFFull) |
+         ((ask >> (p & 63)) & 1 ? 0ull : 0xFFFFFFFFull << 32);
+}
+
+__global__ __launch_bounds__(256) void live_levels_kernel(Book b, int32_t W, int64_t m, uint64_t *out) {
+  const int32_t p = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (p < b.L) out[p] = live_level(b, W, m, p);
+}
+
+// Where a market's levels are left for the host: pinned memory of the calling host
+// thread, allocated on its first use and freed when the thread ends.
+struct HostLevels {
+  uint64_t *p = nullptr;
+  ~HostLevels() { rt_free_pinned(p); }
+};
+
+// One market's book on the host: its levels {bid head, bid tail, ask head, ask tail}
+// (valid until this thread's next call) and its order records. Waits for the stream.
+// The mask words that say which levels are empty lie M apart: copied to the host one by
+// one, at about 11 us each, they made to_string 88 us at 128 levels and 440 at 1,024 (a
+// strided copy is as slow from 16 words on). A kernel that applies them and writes to
+// pinned memory takes the place of the level words' copy too: 36 and 40 us.
+int read_book(const astra_market *h, int32_t market_id, const uint16_t *&levels,
+              std::vector<uint4> &rec, hipStream_t st) {
+  static thread_local HostLevels host;
+  if (!host.p)
+    ASTRA_HIP_CHECK(rt_alloc_pinned(&host.p, ASTRA_EXT_MAX_PRICE_LEVELS * sizeof(uint64_t)), "ToString");
+  const Book b = book_of(h);
+  ASTRA_HIP_CHECK(rt_memcpy(rec.data(), b.records + (size_t)market_id * h->O, (size_t)h->O * 16, st),
+                  "ToString");
+  if (h->L > 0) {
+#ifdef ASTRA_HOST_EMULATION
+    for (int32_t p = 0; p < h->L; ++p) host.p[p] = live_level(b, h->lay.W, market_id, p);
+#else
+    // (the last thing enqueued: no return leaves it running, to write into a later call's levels)
+    hipLaunchKernelGGL(live_levels_kernel, dim3(grid_for(h->L, 256)), dim3(256), 0, st, b, h->lay.W,
+                       (int64_t)market_id, host.p);
+#endif
+    ASTRA_HIP_CHECK(rt_last_error(), "ToString");
+  }
+  ASTRA_HIP_CHECK(rt_sync(st), "ToString");
+  levels = reinterpret_cast<const uint16_t *>(host.p);
+  return ASTRA_OK;
+}
+
 // The TID counter's advance of a call on zero markets, which launches no
 // matching kernel (the reference moves its counter on whatever M is).
 int advance_tid_empty(astra_market *h, int32_t by, hipStream_t s) {
@@ -3010,32 +3060,17 @@ int astra_market_to_string(const astra_market *h, int32_t market_id, char *buf, 
     s = line;
   } else {
     DeviceGuard g(h->device);
-    std::vector<uint16_t> lv((size_t)h->L * 4);
+    const uint16_t *lv = nullptr;
     std::vector<uint4> rec((size_t)h->O);
-    std::vector<uint64_t> masks((size_t)2 * h->lay.W);
-    hipStream_t st = as_stream(stream);
-    if (h->L > 0)
-      ASTRA_HIP_CHECK(rt_memcpy(lv.data(), h->ws + h->lay.levels + (size_t)market_id * h->L * 8,
-                                (size_t)h->L * 8, st),
-                      "ToString");
-    ASTRA_HIP_CHECK(rt_memcpy(rec.data(), h->ws + h->lay.records + (size_t)market_id * h->O * 16,
-                              (size_t)h->O * 16, st),
-                    "ToString");
-    for (size_t i = 0; i < masks.size(); ++i)
-      ASTRA_HIP_CHECK(rt_memcpy(&masks[i], h->ws + h->lay.masks + (i * h->M + market_id) * 8, 8, st),
-                      "ToString");
-    ASTRA_HIP_CHECK(rt_sync(st), "ToString");
+    const int rc = read_book(h, market_id, lv, rec, as_stream(stream));
+    if (rc) return rc;
     std::vector<Row> sells, buys;
-    // the head of level p's list on `side`: its word counts where the mask bit is set
-    auto head = [&](int32_t p, int side) -> uint32_t {
-      return (masks[(size_t)(side * h->lay.W + p / 64)] >> (p % 64)) & 1 ? lv[(size_t)p * 4 + 2 * side] : kNull16;
-    };
-    for (int32_t p = 0; p < h->L; ++p) walk_level(rec, head(p, 1), p, h->O, sells);
+    for (int32_t p = 0; p < h->L; ++p) walk_level(rec, lv[(size_t)p * 4 + 2], p, h->O, sells);
     std::sort(sells.begin(), sells.end(), [](const Row &a, const Row &b) {  // :645-651
       if (a.price != b.price) return a.price > b.price;
       return a.tid < b.tid;
     });
-    for (int32_t p = h->L - 1; p >= 0; --p) walk_level(rec, head(p, 0), p, h->O, buys);
+    for (int32_t p = h->L - 1; p >= 0; --p) walk_level(rec, lv[(size_t)p * 4], p, h->O, buys);
     std::snprintf(line, sizeof line, "####### %zu sell orders #######\n", sells.size());  // :677
     s += line;
     for (const Row &r : sells) {

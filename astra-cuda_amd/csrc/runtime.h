@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
 #include <string>
 
@@ -35,6 +36,11 @@ inline hipError_t rt_memcpy(void *d, const void *s, size_t n, hipStream_t) {
   return hipSuccess;
 }
 inline hipError_t rt_sync(hipStream_t) { return hipSuccess; }
+inline hipError_t rt_alloc_pinned(uint64_t **p, size_t n) {
+  *p = static_cast<uint64_t *>(std::malloc(n));
+  return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+inline void rt_free_pinned(uint64_t *p) { std::free(p); }
 inline hipError_t rt_last_error() { return hipSuccess; }
 // The host build stands in for gfx950: 256 CUs with 160 KB of LDS each, all of
 // which one workgroup may use.
@@ -66,6 +72,25 @@ inline hipError_t rt_memcpy(void *d, const void *s, size_t n, hipStream_t st) {
   return hipMemcpyAsync(d, s, n, hipMemcpyDefault, st);
 }
 inline hipError_t rt_sync(hipStream_t st) { return hipStreamSynchronize(st); }
+// Lets the calling thread allocate and free while a stream captures, whose capture that
+// would end otherwise.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  hipError_t e;
+  RelaxedCapture() : e(hipThreadExchangeStreamCaptureMode(&mode)) {}
+  ~RelaxedCapture() {
+    if (e == hipSuccess) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+};
+// Host memory that kernels on any device may write.
+inline hipError_t rt_alloc_pinned(uint64_t **p, size_t n) {
+  RelaxedCapture relaxed;
+  return hipHostMalloc(reinterpret_cast<void **>(p), n, hipHostMallocPortable);
+}
+inline void rt_free_pinned(uint64_t *p) {
+  RelaxedCapture relaxed;
+  if (p) (void)hipHostFree(p);
+}
 inline hipError_t rt_last_error() { return hipGetLastError(); }
 inline hipError_t rt_lds_per_block(int dev, int *bytes) {
   return hipDeviceGetAttribute(bytes, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);

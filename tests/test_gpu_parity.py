@@ -309,6 +309,61 @@ def test_gpu_reset_clear_clone_and_to_string():
     compare_portfolios(g, o, "original after clone")
 
 
+def test_gpu_to_string_cost_and_threads():
+    """A market's mask words lie M apart; to_string must not pay a copy for each of them:
+    1,024 levels (32 words) within twice the time of 64 levels (2 words), at their fastest,
+    where a copy per word takes six times as long. Every thread reads its own book, and a
+    thread's first call does not end a capture that goes on elsewhere."""
+    import threading
+    import time
+    from oracle.oracle import OracleMarket
+    from astra_cuda import order_matching as aom
+    M, O, F, C = 300, 64, 64, 4
+    books, best = [], []
+    for L in (64, 1024):
+        g, o = aom.VecMarket(M, L, O, F, C, allow_extended_shapes=True), OracleMarket(M, L, O, F, C)
+        gf, of = g.new_fill_batch(), o.new_fill_batch()
+        rng = np.random.default_rng(L)
+        for _ in range(20):
+            q = [rng.integers(0, L, M), rng.integers(0, 5, M), rng.integers(0, L, M), rng.integers(0, 5, M),
+                 rng.integers(0, C, M)]
+            q = [a.astype(np.int32) for a in q]
+            g.add_two_sided_quotes(*(t32(a) for a in q), gf)
+            o.add_two_sided_quotes(*q, of)
+        books.append((g, [o.to_string(m) for m in range(M)]))
+        times = []
+        for m in range(40):
+            t = time.perf_counter()
+            g.to_string(m)
+            times.append(time.perf_counter() - t)
+        best.append(min(times))
+    print(f"to_string: {best[0] * 1e6:.1f} us at 64 levels, {best[1] * 1e6:.1f} at 1,024", flush=True)
+    wrong = []
+
+    def read(side, g, texts, rounds):
+        with torch.cuda.stream(side):
+            wrong.extend(m for _ in range(rounds) for m in range(M) if g.to_string(m) != texts[m])
+
+    threads = [threading.Thread(target=read, args=(torch.cuda.Stream(), *books[i % 2], 2)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    x, graph, side = torch.zeros(8, device=DEV), torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, capture_error_mode="thread_local"):
+        x.add_(1)
+        first = threading.Thread(target=read, args=(side, *books[0], 1))
+        first.start()
+        first.join()
+        x.add_(1)
+    for k in range(1, 4):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert x.tolist() == [2.0 * k] * 8
+    assert not wrong, wrong[:10]
+    assert best[1] < 2 * best[0], best
+
+
 @pytest.mark.parametrize("M", [1, 64, 257, 4000])
 @pytest.mark.parametrize("L", [1, 64, 65, 129, 513])
 def test_gpu_emptied_and_cleared_levels_start_anew(L, M):

@@ -1290,7 +1290,7 @@ ASTRA_HD bool zero_levels(LoopState<W> &s, const MarketCtx &c, const BookMem &bk
 // instruction issue, taken branches and LDS round trips one after another);
 // this run keeps its state in registers, reads both head records together
 // once per pass, and writes a surviving order's size and a level's new head
-// once, when the run ends or the level empties. Called at the top of a pass
+// once, when the run ends (a level that empties has none). Called at the top of a pass
 // with both records loaded and the book crossing; returns whether it made a
 // pass, and leaves every write in the book and the state at the top of a pass
 // (the loop's next pass reads both records again).
@@ -1325,8 +1325,7 @@ ASTRA_HD bool cross_run(LoopState<W> &s, const MarketCtx &c, const BookMem &bk, 
     if (pop_b) {
       bk.set_size(s.bh, 0);
       if (nb == kNull16) {
-        if (head_b) bk.set_head(s.bb, 0, s.bh);  // what the passes one by one leave
-        head_b = false;
+        head_b = false;  // the word of an empty level is not read
         mask_clear<W>(s.bm, s.bb);
         if (STATS) ++s.emptied;
         s.bb = mask_highest<W>(s.bm);
@@ -1341,7 +1340,6 @@ ASTRA_HD bool cross_run(LoopState<W> &s, const MarketCtx &c, const BookMem &bk, 
     if (pop_a) {
       bk.set_size(s.ah, 0);
       if (na == kNull16) {
-        if (head_a) bk.set_head(s.ba, 1, s.ah);  // what the passes one by one leave
         head_a = false;
         mask_clear<W>(s.am, s.ba);
         if (STATS) ++s.emptied;

@@ -241,6 +241,76 @@ def test_emulated_emptied_and_cleared_levels_start_anew(L):
                 assert e.to_string(m) == o.to_string(m), (L, t, m)
 
 
+def _words(e, L):
+    """The level words of an emulated market: uint16 [M, L, {bid head, tail, ask head, tail}]."""
+    from ws_layout import layout
+    o, n = layout(e.M, L, e.O, e.C)["levels"]
+    return e.ws[o:o + n].view(np.uint16).reshape(e.M, L, 4)
+
+
+@pytest.mark.parametrize("stage_budget", [None, 1])
+@pytest.mark.parametrize("L", [1, 65, 128, 513])
+def test_emulated_empty_levels_hold_any_word(L, stage_budget):
+    """Before every call the words of the empty levels are overwritten with slots of the
+    ring, which a missing look at the mask bit would take for orders (exact)."""
+    from ws_layout import layout, mask_words
+    M, O, F, C = 33, 24, 30, 3
+    rng = np.random.default_rng(100 + L)
+    e, o = _emu(M, L, O, F, C, stage_budget, extended=True), OracleMarket(M, L, O, F, C)
+    ef, of = e.new_fill_batch(), o.new_fill_batch()
+    eb, ob = e.new_bbo_batch(), o.new_bbo_batch()
+    words = _words(e, L)
+    at, n = layout(M, L, O, C)["masks"]
+    masks = e.ws[at:at + n].view(np.uint64).reshape(2, mask_words(L), M)
+    for t in range(150):
+        bits = np.ascontiguousarray(masks.transpose(2, 0, 1)).view(np.uint8)
+        empty = np.unpackbits(bits, axis=2, count=L, bitorder="little").transpose(0, 2, 1) == 0  # [M, L, 2]
+        words[np.repeat(empty, 2, axis=2)] = rng.integers(0, O, 2 * int(empty.sum())).astype(np.uint16)
+        lo = rng.integers(0, L, M)
+        args = (lo, rng.integers(0, 4, M), np.clip(lo + rng.integers(-2, 3, M), 0, L - 1), rng.integers(0, 4, M),
+                rng.integers(0, C, M))
+        args = [a.astype(np.int32) for a in args]
+        e.add_two_sided_quotes(*args, ef)
+        o.add_two_sided_quotes(*args, of)
+        if t % 5 == 3:
+            mask = rng.random(M) < 0.4
+            e.clear_quotes(mask)
+            o.clear_quotes(mask)
+        if t == 90:
+            e.reset()
+            o.reset()
+        e.get_bbos(eb)
+        o.get_bbos(ob)
+        _compare(e, ef, eb, o, of, ob, F, f"L={L} step {t}")
+        for m in range(t % 4, M, 4):
+            assert e.to_string(m) == o.to_string(m), (L, t, m)
+
+
+@pytest.mark.parametrize("side", [0, 1])
+def test_emulated_a_run_that_empties_a_level_leaves_its_word(side):
+    """Three orders at a level and one quote that takes them all: the first pass moves the
+    level's head to the second order, and the run on the staged book, which moves on to
+    the third and past it, writes nothing more to the level that it empties."""
+    from ws_layout import layout
+    L, O, px = 8, 64, 4
+    e = _emu(1, L, O, 16, 2, stage_budget=1)
+    f = e.new_fill_batch()
+    one = np.ones(1, np.int32)
+
+    def quote(bid, ask):  # sizes; 0 places no order
+        e.add_two_sided_quotes(one * px, one * bid, one * px, one * ask, one, f)
+
+    for _ in range(3):
+        quote(*((0, 1) if side else (1, 0)))
+    word = _words(e, L)[0, px]
+    first, last = word[2 * side], word[2 * side + 1]
+    at, n = layout(1, L, O, 2)["records"]
+    second = e.ws[at:at + n].view(np.uint32).reshape(O, 4)[first, 3] >> 16  # {.., price | next << 16}
+    quote(*((3, 0) if side else (0, 3)))
+    assert f.fill_counts[0] == 3
+    assert (word[2 * side], word[2 * side + 1]) == (second, last)
+
+
 def test_emulated_zero_sized_shapes():
     # M = 0 and F = 0 and L = 0 are accepted by the reference constructor
     em = EmuMarket(0, 128, 16, 16, 4)

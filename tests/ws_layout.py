@@ -7,7 +7,9 @@ hands out as a BBO, single calls only those whose order record they hold in
 registers (get_bbos reads the others from the book, so both give the same
 BBOs). ``normalized`` clears the cache's flags (bit 15 of each half of the tob
 word that holds a slot; an empty head, 0xFFFF, keeps its value) and its size
-array, leaving everything else as it is.
+array. Nor has an empty level's word a value (its mask bit says that it is empty,
+and what its last orders left there is not read): ``normalized`` sets both words of
+each side without its bit to NULL. Everything else stays as it is.
 
 The workspace starts with 256 bytes of control words (int32): the TID counter
 of a book with no markets (otherwise every market keeps a copy in ``tids``) and
@@ -43,21 +45,23 @@ def layout(M: int, L: int, O: int, C: int) -> dict:
 
 def normalized(ws, M: int, L: int, O: int, C: int):
     """A copy of the workspace bytes (a numpy or torch uint8 array) with the
-    head-size cache cleared."""
+    head-size cache cleared and the empty levels' words NULL."""
     import numpy as np
-    is_np = isinstance(ws, np.ndarray)
-    w = ws.copy() if is_np else ws.clone()
-    lay = layout(M, L, O, C)
-    o, n = lay["tob"]
-    if n:
-        # bit 15 of a half flags a cached size; 0xFFFF (empty) carries no flag
-        if is_np:
-            h = w[o:o + n].view(np.uint16)
-            h[h != 0xFFFF] &= 0x7FFF
-        else:
-            import torch
-            h = w[o:o + n].view(torch.int16)
-            h.copy_(torch.where(h == -1, h, h & 0x7FFF))
-    o, n = lay["hsz"]
-    w[o:o + n] = 0
+    if not isinstance(ws, np.ndarray):
+        import torch
+        return torch.from_numpy(normalized(ws.cpu().numpy(), M, L, O, C))
+    w, lay = ws.copy(), layout(M, L, O, C)
+
+    def array(name, dtype):
+        o, n = lay[name]
+        return w[o:o + n].view(dtype)
+
+    # bit 15 of a half flags a cached size; 0xFFFF (empty) carries no flag
+    h = array("tob", np.uint16)
+    h[h != 0xFFFF] &= 0x7FFF
+    array("hsz", np.uint8)[:] = 0
+    bits = array("masks", np.uint64).reshape(2, mask_words(L), M).transpose(2, 0, 1)
+    bits = np.ascontiguousarray(bits).view(np.uint8)
+    live = np.unpackbits(bits, axis=2, count=L, bitorder="little").transpose(0, 2, 1)  # [M, L, 2]
+    array("levels", np.uint32).reshape(M, L, 2)[live == 0] = 0xFFFFFFFF  # {head, tail} of a side
     return w

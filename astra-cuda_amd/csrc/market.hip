@@ -2623,9 +2623,9 @@ int advance_tid_empty(astra_market *h, int32_t by, hipStream_t s) {
   return ASTRA_OK;
 }
 
-// Empty book: TID counter 0, masks 0, slot counters 0, BBO cache empty, level
-// words NULL, portfolios 0 (the
-// order records are left alone: no list reaches a slot before it is written).
+// Empty book: TID counter 0, masks 0, slot counters 0, BBO cache empty, portfolios 0.
+// Level words and order records are left alone: an empty level's word is not read, and no
+// list reaches a slot before it is written.
 int init_book(astra_market *h, hipStream_t s) {
   const Layout &l = h->lay;
   int rc;
@@ -2635,8 +2635,6 @@ int init_book(astra_market *h, hipStream_t s) {
   int32_t *bbo = reinterpret_cast<int32_t *>(h->ws + l.bbo);
   if ((rc = launch_fill(bbo, 2 * (int64_t)h->M, 0xFFFFFFFFu, s, "init"))) return rc;
   if ((rc = launch_fill(h->ws + l.tob, h->M, 0xFFFFFFFFu, s, "init"))) return rc;
-  if ((rc = launch_fill(h->ws + l.levels, (int64_t)h->M * h->L * 2, 0xFFFFFFFFu, s, "init")))
-    return rc;
   return launch_fill(h->ws + l.portfolios, (int64_t)h->M * h->C * 2, 0u, s, "init");
 }
 
@@ -2809,7 +2807,7 @@ int astra_market_create(int32_t M, int32_t L, int32_t O, int32_t F, int32_t C, i
   h->ws_bytes = workspace_bytes;
   h->lay = lay;
   // the whole workspace to 0 once (order records and alignment padding included, so a
-  // fresh workspace holds no garbage), then the empty book's NULL words
+  // fresh workspace holds no garbage), then the empty book's BBO cache
   rc = launch_fill(h->ws, (int64_t)(lay.total / 4), 0u, as_stream(stream), "init");
   if (!rc) rc = init_book(h, as_stream(stream));
   if (rc) {

@@ -286,6 +286,21 @@ def test_emulated_empty_levels_hold_any_word(L, stage_budget):
             assert e.to_string(m) == o.to_string(m), (L, t, m)
 
 
+def test_emulated_reset_and_clear_leave_the_level_words():
+    """8 bytes per level and market that a reset or a clear need not write (whatever they
+    hold, see above)."""
+    M, L, O = 5, 70, 16
+    e = _emu(M, L, O, 8, 3)
+    words = _words(e, L)
+    words[:] = np.random.default_rng(1).integers(0, O, words.shape)
+    before = words.copy()
+    e.clear_quotes(np.ones(M, bool))
+    assert np.array_equal(words, before)
+    e.reset()
+    assert np.array_equal(words, before)
+    assert e.to_string(4) == OracleMarket(M, L, O, 8, 3).to_string(4)
+
+
 @pytest.mark.parametrize("side", [0, 1])
 def test_emulated_a_run_that_empties_a_level_leaves_its_word(side):
     """Three orders at a level and one quote that takes them all: the first pass moves the

@@ -1788,13 +1788,6 @@ __device__ __forceinline__ T *in_vgpr(T *p) {
 // all the words hold the same value, the reference's counter; no lane waits on
 // another and a captured launch replays with advancing TIDs.
 
-// The counter's advance of a call on zero markets (no matching launch).
-__global__ void tid_advance_kernel(int32_t *ctl, int32_t by) {
-  if (threadIdx.x == 0)
-    __hip_atomic_store(ctl + kCtlTid, (int32_t)((uint32_t)ctl[kCtlTid] + (uint32_t)by),
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Writes the rows owed by fast-forwarded markets of this wavefront: each such
 // lane's rows are written by all 64 lanes together, coalesced.
 __device__ __forceinline__ void write_bulk_wave(const FillOut &out, const Bulk &bk) {
@@ -2198,19 +2191,6 @@ __global__ __launch_bounds__(256) void quote_match_kernel(Book b, QuoteIn in, Fi
   }
 }
 
-__global__ __launch_bounds__(256) void bbo_kernel(Book b, int32_t *bid_px, int32_t *bid_sz,
-                                                  int32_t *ask_px, int32_t *ask_sz) {
-  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (m < b.M) bbo_copy_market(b, bid_px, bid_sz, ask_px, ask_sz, m);
-}
-
-__global__ __launch_bounds__(256) void last_price_kernel(int32_t *last, const int32_t *counts,
-                                                         const int32_t *prices, int32_t M,
-                                                         int32_t F, int32_t stride) {
-  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (m < M) last_price_market(last, counts, prices, F, stride, m);
-}
-
 // One lane per market, coalesced words only (a lane per level, with a 64-bit division
 // to find its market, made a step of 30,000 markets with 1/64 of them cleared 39.7 us;
 // 33.4 us now).
@@ -2218,18 +2198,6 @@ template <int W>
 __global__ __launch_bounds__(256) void clear_quotes_kernel(Book b, const uint8_t *reset) {
   const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (m < b.M) clear_quotes_market<W>(b, reset, m);
-}
-
-// Grid-stride fill of n 32-bit words; 16-byte stores when dst is 16-byte aligned.
-__global__ __launch_bounds__(kFillThreads) void fill_u32_kernel(uint32_t *dst, int64_t n,
-                                                                uint32_t v, int vec) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n4 = vec ? n / 4 : 0;
-  uint4 *d4 = reinterpret_cast<uint4 *>(dst);
-  const uint4 v4 = make_uint4(v, v, v, v);
-  for (int64_t i = t; i < n4; i += stride) d4[i] = v4;
-  for (int64_t i = n4 * 4 + t; i < n; i += stride) dst[i] = v;
 }
 
 // ---- launchers (kernel on the device build, host loop on the emulation build) ----
@@ -2514,6 +2482,40 @@ int launch_for_levels(const Call &c) {
     case 8: return ASTRA_CALL_W(8);
     default: return ASTRA_CALL_W(16);
   }
+}
+
+// ---- kernels that do not depend on W, and their launchers ----
+
+__global__ __launch_bounds__(256) void bbo_kernel(Book b, int32_t *bid_px, int32_t *bid_sz,
+                                                  int32_t *ask_px, int32_t *ask_sz) {
+  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (m < b.M) bbo_copy_market(b, bid_px, bid_sz, ask_px, ask_sz, m);
+}
+
+__global__ __launch_bounds__(256) void last_price_kernel(int32_t *last, const int32_t *counts,
+                                                         const int32_t *prices, int32_t M,
+                                                         int32_t F, int32_t stride) {
+  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (m < M) last_price_market(last, counts, prices, F, stride, m);
+}
+
+// Grid-stride fill of n 32-bit words; 16-byte stores when dst is 16-byte aligned.
+__global__ __launch_bounds__(kFillThreads) void fill_u32_kernel(uint32_t *dst, int64_t n,
+                                                                uint32_t v, int vec) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t n4 = vec ? n / 4 : 0;
+  uint4 *d4 = reinterpret_cast<uint4 *>(dst);
+  const uint4 v4 = make_uint4(v, v, v, v);
+  for (int64_t i = t; i < n4; i += stride) d4[i] = v4;
+  for (int64_t i = n4 * 4 + t; i < n; i += stride) dst[i] = v;
+}
+
+// The counter's advance of a call on zero markets (no matching launch).
+__global__ void tid_advance_kernel(int32_t *ctl, int32_t by) {
+  if (threadIdx.x == 0)
+    __hip_atomic_store(ctl + kCtlTid, (int32_t)((uint32_t)ctl[kCtlTid] + (uint32_t)by),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 int launch_bbo(const astra_market *h, int32_t *bp, int32_t *bs, int32_t *ap, int32_t *as,

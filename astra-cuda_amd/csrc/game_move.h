@@ -218,10 +218,15 @@ ASTRA_HD void game_after(const GameMove &g, const GameQuote &q, const int32_t *p
   // One uniform branch on the player count: with the count a constant no load is
   // made for a player that does not exist, and an env's consecutive words go 16
   // bytes at a time (48 loads of 4 bytes per lane, 18 of them repeats, become 12 at 5
-  // players). An episode of 262,144 envs (40 moves) 3.86 -> 3.73 ms; what bounds the
-  // move there is the two wavefronts per SIMD its 220-256 registers allow. Kept under
-  // 168 registers, for three, it spills and takes 4.08 ms. Other counts (below 4, above
-  // 8) go four at a time.
+  // players). A move of 65,536 envs 33.0 -> 28.7 us, an episode of 262,144 (40 moves)
+  // 3.86 -> 3.73 ms; what bounds the move there is the two wavefronts per SIMD its 220-256
+  // registers allow. Kept under 168 registers, for three, it spills and takes 4.08 ms.
+  // Other counts (below 4, above 8) go four at a time, which beats a clamped batch of eight
+  // though it makes more round trips: with eight the kernel needs 24-44 registers beyond
+  // 256 and one wavefront per SIMD is left. A move of 65,536 envs and 9 players takes 36.7
+  // us so, 44.6 with eight (and 5 players 35.8); 12 players 41.6 and 50.3, an episode of 16
+  // players 12.1 and 12.5 ms. Before the counts were written out they took 42.2, 47.4 and
+  // 12.7.
   switch (P) {
     case 4: return game_players<4, true>(g, pf_m, M, m, pc, 0, charge, settle, value);
     case 5: return game_players<5, true>(g, pf_m, M, m, pc, 0, charge, settle, value);

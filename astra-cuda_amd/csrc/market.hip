@@ -1066,10 +1066,10 @@ ASTRA_HD void quote_prologue(const Book &b, const QuoteIn &in, int64_t m, Market
   // here, while the masks are at hand, not behind the second round trip. A pop that
   // empties a level and ClearQuotes then store no NULL word (one scattered write of
   // about 17 per market and step less; large launches are bound by such requests).
-  // Steps of one state after another, past the ring's wrap: 524,288 markets 371 ->
-  // 360 us, 16 steps of 100,000 in one launch (row layout) 626 -> 611, 32 of 10,000
-  // 357 -> 350, 100,000 markets 65.8 -> 63.5 (with the select 68.7, with the OR behind
-  // the second round trip 66.7) and unchanged where states alternate.
+  // Steps past the ring's wrap, medians of four alternating runs: 524,288 markets 375 ->
+  // 371 us, 16 steps of 100,000 in one launch (row layout) 647 -> 637, 100,000 markets
+  // 66.2 -> 63.3 (in one sweep of 65.8 before and 63.5 so, the select gave 68.7 and the OR
+  // behind the second round trip 66.7). 10,000 to 33,333 markets: within 1%.
   const uint32_t bnone = pinned(mask_absent<W>(s.bm, bid_px));
   const uint32_t anone = pinned(mask_absent<W>(s.am, ask_px));
 
@@ -2191,9 +2191,9 @@ __global__ __launch_bounds__(256) void quote_match_kernel(Book b, QuoteIn in, Fi
   }
 }
 
-// One lane per market, coalesced words only (a lane per level, with a 64-bit division
-// to find its market, made a step of 30,000 markets with 1/64 of them cleared 39.7 us;
-// 33.4 us now).
+// One lane per market, coalesced words only: 2.6 us for 30,000 markets of 128 levels, 1/64
+// of them cleared (a lane per level, with a 64-bit division to find its market and a NULL
+// word to store, took 6.5; the step of five launches around it 37.4 -> 33.3 us).
 template <int W>
 __global__ __launch_bounds__(256) void clear_quotes_kernel(Book b, const uint8_t *reset) {
   const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
